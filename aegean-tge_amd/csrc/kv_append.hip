@@ -47,6 +47,124 @@ __global__ __launch_bounds__(256) void kv_append_kernel(AppendParams p) {
   store_lane<FMT>(p, x, p.rows[row], which, h, b, quarter, live);
 }
 
+// Append by page, for steps of many rows: a wave owns 64 lane tasks of one
+// page block, each 4 consecutive token slots x 8 dims of K or V, so that
+// they make up one contiguous run of 2048 elements of the block (128-dim
+// blocks: K or V; 256: a half of K or V). A whole page's codes are put into
+// the block's order in the wave's LDS and leave as 16-byte pieces, one
+// contiguous KiB per store. Pages that the step writes in part store element
+// by element, as the row kernel does.
+// Bound by memory once the chip is full (the row kernel by its 1- and 2-byte
+// V stores). 20,000 rows, row kernel -> this one: 4 heads of 128 dims int8
+// 38.8 -> 28.5 us (104 MB), f16 44.7 -> 27.9 us (123 MB: 4.4 TB/s); 8 heads
+// of 256 dims int8 174 -> 88 us, f16 226 -> 91 us (491 MB: 5.4 TB/s).
+template <int FMT>
+__global__ __launch_bounds__(256) void kv_append_pages_kernel(AppendParams p) {
+  constexpr int E = FMT == kF16 ? 2 : 1;
+  constexpr int kRun = 2048 * E;  // bytes of a wave's run
+  __shared__ __align__(16) char stage[4][kRun];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nb = p.head_dim >> 5, runs = nb >> 1;  // 4 or 8 blocks of 32; 2 or 4 runs
+  const long unit = (long)blockIdx.x * 4 + wave;
+  if (unit >= (long)p.n_tiles * p.kv_heads * runs) return;  // whole waves
+  const int run = (int)(unit & (runs - 1));
+  const long rest = unit / runs;
+  const int h = (int)(rest % p.kv_heads);
+  const TileRec t = p.tiles[rest / p.kv_heads];
+
+  // Lane -> (slots 4g.., block, quarter): the four lanes of a 32-value block
+  // are adjacent, and 16 lanes read 512 bytes of one token's row.
+  const int which = run >= runs / 2;
+  const int quarter = lane & 3, g = lane >> 4;
+  const int b = (run - (which ? runs / 2 : 0)) * 4 + ((lane >> 2) & 3);
+  const int d0 = b * 32 + quarter * 8;
+
+  float x[4][8];
+  const size_t row_len = (size_t)p.kv_heads * p.dims;
+  const float* src = (which ? p.v : p.k) + (size_t)h * p.dims;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    // (slots without a row read the nearest one and are not stored)
+    const int i = min(max(4 * g + j - t.slot, 0), t.count - 1);
+    const float* head_row = src + (size_t)(t.row + i) * row_len;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[j][e] = 0.0f;  // (dims past the head's own)
+    if ((p.dims & 7) == 0) {
+      if (d0 < p.dims) load8(x[j], head_row + d0);
+    } else {
+      load8_head(x[j], head_row, d0, p.dims);
+    }
+  }
+  LaneCodes c[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) c[j] = encode_lane<FMT>(x[j]);
+
+  char* const blk = static_cast<char*>(p.pool) + ((size_t)t.page * p.kv_heads + h) * p.geom.block_bytes;
+  if (t.count < kPageTokens) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int slot = 4 * g + j;
+      if (slot >= t.slot && slot < t.slot + t.count)
+        write_lane<FMT>(GlobalPut{blk}, p.geom, nb, p.scale_f32 != 0, c[j], slot, which, b, quarter);
+    }
+    return;
+  }
+
+  char* const st = stage[wave];
+  const int base = run * kRun - (which ? p.geom.v_off() : 0);  // the run's start in the part
+  if (which == 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int k0 = k_index(4 * g + j, d0, E) * E - base;
+      const int k1 = k_index(4 * g + j, d0 + 4, E) * E - base;
+      if (FMT == kF16) {
+        *reinterpret_cast<uint2*>(st + k0) = make_uint2(c[j].w[0], c[j].w[1]);
+        *reinterpret_cast<uint2*>(st + k1) = make_uint2(c[j].w[2], c[j].w[3]);
+      } else {
+        *reinterpret_cast<uint32_t*>(st + k0) = c[j].w[0];
+        *reinterpret_cast<uint32_t*>(st + k1) = c[j].w[1];
+      }
+    }
+  } else {
+    // one dim's four tokens are adjacent in the V part
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int off = v_index(4 * g, d0 + i, E) * E - base;
+      if (FMT == kF16) {
+        uint32_t e[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e[j] = (c[j].w[i >> 1] >> (16 * (i & 1))) & 0xffffu;
+        *reinterpret_cast<uint2*>(st + off) = make_uint2(e[0] | e[1] << 16, e[2] | e[3] << 16);
+      } else {
+        uint32_t v = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v |= ((c[j].w[i >> 2] >> (8 * (i & 3))) & 0xffu) << (8 * j);
+        *reinterpret_cast<uint32_t*>(st + off) = v;
+      }
+    }
+  }
+  if (FMT != kF16 && quarter == 0) {  // the block's scales of four tokens are adjacent
+    char* const sp = blk + (which ? p.geom.vs_off() : p.geom.ks_off());
+    const int si = scale_index_np(4 * g, b, nb);
+    if (p.scale_f32) {
+      *reinterpret_cast<float4*>(sp + si * 4) = make_float4(c[0].scale, c[1].scale, c[2].scale, c[3].scale);
+    } else {
+      uint32_t e[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) e[j] = float_to_half_ref(c[j].scale);
+      *reinterpret_cast<uint2*>(sp + si * 2) = make_uint2(e[0] | e[1] << 16, e[2] | e[3] << 16);
+    }
+  }
+  // the wave's own LDS: its writes are ordered before its reads
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int i = 0; i < kRun / 1024; ++i)
+    *reinterpret_cast<uint4*>(blk + run * kRun + i * 1024 + lane * 16) =
+        *reinterpret_cast<const uint4*>(st + i * 1024 + lane * 16);
+}
+
 // NeoX rotation of one (low, high) pair by (c, s), in the rounding of
 // apply_rope_avx2 (attention's default CPU path: l*c - (h*s) and
 // l*s + (h*c) with one rounding each, norm_rope_avx2.cpp:97-131) or of
@@ -207,6 +325,16 @@ __global__ __launch_bounds__(256) void kv_gather_kernel(GatherParams p) {
 hipError_t launch_kv_append(int format, const AppendParams& p, hipStream_t stream) {
   const long total = (long)p.n_rows * 2 * p.kv_heads * (p.head_dim >> 5) * 4;
   if (total == 0) return hipSuccess;
+  if (p.tiles) {
+    const long units = (long)p.n_tiles * p.kv_heads * (p.head_dim >> 6);
+    const dim3 grid((unsigned)((units + 3) / 4)), block(256);
+    if (format == kF16) {
+      hipLaunchKernelGGL(kv_append_pages_kernel<kF16>, grid, block, 0, stream, p);
+    } else {
+      hipLaunchKernelGGL(kv_append_pages_kernel<kI8>, grid, block, 0, stream, p);
+    }
+    return hipGetLastError();
+  }
   const dim3 grid((unsigned)((total + 255) / 256)), block(256);
   if (format == kF16) {
     hipLaunchKernelGGL(kv_append_kernel<kF16>, grid, block, 0, stream, p);

@@ -193,7 +193,8 @@ struct tge_batch {
 
   // Device image: sessions | tables | rows (one allocation), pinned staging.
   tge::plan::Staged image;
-  size_t off_sessions = 0, off_tables = 0, off_rows = 0;
+  size_t off_sessions = 0, off_tables = 0, off_rows = 0, off_tiles = 0;
+  std::vector<tge::TileRec> tiles;  // the append's, by page (empty: row by row)
 
   // Kernel timing (tge_batch_set_profiling): per attention call since
   // enabling, events before the attention kernel, between it and the merge,
@@ -504,7 +505,7 @@ int tge_batch_plan(tge_batch* b, const tge_kv_pool* pool, const tge_batch_desc* 
 
   hipStream_t hs = static_cast<hipStream_t>(stream);
   // The step's lists are built on the host first and go up in one copy:
-  // [ sessions | tables | rows | attention lists | step records |
+  // [ sessions | tables | rows | append tiles | attention lists | step records |
   // first-batch page ids ]. The attention lists are the decode lists when
   // every session's rows fit a decode unit (one upload per step serves every
   // layer), the block-prefill lists when none does (a prompt chunk); a step
@@ -527,7 +528,9 @@ int tge_batch_plan(tge_batch* b, const tge_kv_pool* pool, const tge_batch_desc* 
   const size_t o_sess = 0;
   const size_t o_tab = align_up(o_sess + st.sessions.size() * sizeof(tge::SessionRec));
   const size_t o_rows = align_up(o_tab + st.tables.size() * sizeof(int));
-  const size_t o_dec = align_up(o_rows + st.rows.size() * sizeof(tge::RowRec));
+  tge::plan::build_append_tiles(st, b->tiles);
+  const size_t o_tiles = align_up(o_rows + st.rows.size() * sizeof(tge::RowRec));
+  const size_t o_dec = align_up(o_tiles + b->tiles.size() * sizeof(tge::TileRec));
   AttnPlan& dp = dec ? b->decode : b->prefill;  // (the eager attention plan, if any)
   const bool eager = dec || pre;
   const size_t dec_bytes =
@@ -540,6 +543,8 @@ int tge_batch_plan(tge_batch* b, const tge_kv_pool* pool, const tge_batch_desc* 
     std::memcpy(h + o_sess, st.sessions.data(), st.sessions.size() * sizeof(tge::SessionRec));
     if (!st.tables.empty()) std::memcpy(h + o_tab, st.tables.data(), st.tables.size() * sizeof(int));
     std::memcpy(h + o_rows, st.rows.data(), st.rows.size() * sizeof(tge::RowRec));
+    if (!b->tiles.empty())
+      std::memcpy(h + o_tiles, b->tiles.data(), b->tiles.size() * sizeof(tge::TileRec));
     if (eager) tge::plan::write_image(dp.lists, dp.off_reduce, dp.off_first, h + o_dec, dp.off_app);
     if (small) {
       std::memcpy(h + o_step, SL.recs.data(), rbytes);
@@ -550,6 +555,7 @@ int tge_batch_plan(tge_batch* b, const tge_kv_pool* pool, const tge_batch_desc* 
   b->off_sessions = o_sess;
   b->off_tables = o_tab;
   b->off_rows = o_rows;
+  b->off_tiles = o_tiles;
   if (eager) {
     dp.dev = b->image.dev + o_dec;
     s = finish_plan(dp, st.block_dims, hs);
@@ -759,6 +765,10 @@ int tge_kv_append(const tge_batch* b, tge_kv_pool* p, int layer, const float* k,
   a.head_dim = p->bd;
   a.dims = b->step.head_dim;
   a.scale_f32 = p->desc.scale_format == TGE_SCALE_F32;
+  if (!b->tiles.empty()) {
+    a.tiles = reinterpret_cast<const tge::TileRec*>(b->image.dev + b->off_tiles);
+    a.n_tiles = (int)b->tiles.size();
+  }
   TGE_HIP(tge::launch_kv_append(p->desc.format, a, static_cast<hipStream_t>(stream)));
   return TGE_OK;
 }

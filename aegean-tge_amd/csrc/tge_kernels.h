@@ -22,6 +22,10 @@ struct AppendParams {
   int head_dim;  // block width
   int dims;      // the head's dims
   int scale_f32;
+  // Per-page records of the rows (the plan's append tiles): the launch
+  // stores page by page (kv_append_pages_kernel). Null: row by row.
+  const TileRec* tiles;
+  int n_tiles;
   // Fused bias + RoPE (launch_kv_append_rope only): k/v above are the
   // pre-bias, pre-RoPE rows; q (optional) is rotated into q_out.
   const float* q;  // [n_rows][q_heads*dims], or null

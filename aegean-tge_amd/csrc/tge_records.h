@@ -131,4 +131,15 @@ struct RowRec {  // one new token: destination page and slot, logical position
   int pos;
 };
 
+// The new rows of one session that fall into one page: `count` consecutive
+// rows from `row`, at the page's slots `slot` on.
+struct TileRec {
+  int page;
+  int row;
+  int slot;
+  int count;
+};
+
+static_assert(sizeof(TileRec) == 4 * sizeof(int), "TileRec is read as 4 ints");
+
 }  // namespace tge

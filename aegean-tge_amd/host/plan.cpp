@@ -143,6 +143,21 @@ int build_step(Step& step, int ns, const int* ctx, const int* n_new, const int* 
   return TGE_OK;
 }
 
+void build_append_tiles(const Step& s, std::vector<TileRec>& tiles) {
+  tiles.clear();
+  const long lanes = (long)s.rows.size() * 2 * s.kv_heads * (s.block_dims / 8);
+  if (s.block_dims <= 64 || lanes * s.block_dims < kAppendPageWork) return;
+  for (const auto& sr : s.sessions) {
+    for (int j = 0; j < sr.n_new;) {
+      const int slot = (sr.ctx + j) % kPageTokens;
+      const int n = std::min(kPageTokens - slot, sr.n_new - j);
+      tiles.push_back(TileRec{s.rows[(std::size_t)(sr.q_row + j)].page, sr.q_row + j, slot, n});
+      j += n;
+    }
+  }
+  if (s.rows.size() < 12 * tiles.size()) tiles.clear();
+}
+
 bool decode_session(const Step& s, const SessionRec& r) {
   return r.n_new * s.group <= max_unit_rows(s.block_dims);
 }

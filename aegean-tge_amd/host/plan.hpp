@@ -81,6 +81,19 @@ int build_step(Step& step, int n_sessions, const int* ctx, const int* n_new,
                const int* table_offsets, const int* page_ids, int q_heads, int kv_heads,
                int head_dim, int pool_pages, const char** message);
 
+// The step's new rows page by page (TileRec) when its append should store
+// whole pages, empty when it should go row by row. By page a launch has a
+// longer fixed time (four tokens per lane, staged: 5.5-6 us against 4.2) and
+// the better rate, so it takes steps whose lanes (8 values each, in the row
+// kernel) times block width reach 2^26. Row kernel / page kernel, us: 128
+// dims, 4 heads, 2048 rows (2^18 lanes) f16 7.4 / 7.9, int8 6.3 / 6.9; 4096
+// rows 11.6 / 9.2, 9.3 / 8.5; 256 dims, 8 heads, 256 rows (2^17) 6.5 / 7.0,
+// 5.0 / 6.6; 512 rows 9.4 / 7.5, 7.0 / 6.8. 64-dim blocks stay with the row
+// kernel (2 heads, 20,000 rows: int8 9.3 / 10.5), and so do steps whose rows
+// fill their pages to less than three quarters on average.
+constexpr long kAppendPageWork = 1L << 26;
+void build_append_tiles(const Step& s, std::vector<TileRec>& tiles);
+
 // Work lists of one attention kind for the current step.
 struct AttnLists {
   std::vector<WorkRec> work;

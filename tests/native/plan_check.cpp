@@ -182,6 +182,30 @@ void check_lists(const Step& st, const AttnLists& l, int only, bool prefill) {
   }
 }
 
+int append_tiles_seen = 0;
+
+// The append's page records hold every new row once, in order, each
+// record's rows in one page at consecutive slots; none for small steps.
+void check_append_tiles(const Step& st) {
+  std::vector<TileRec> tiles;
+  build_append_tiles(st, tiles);
+  const long lanes = (long)st.rows.size() * 2 * st.kv_heads * (st.block_dims / 8);
+  if (st.block_dims <= 64 || lanes * st.block_dims < kAppendPageWork)
+    REQUIRE(tiles.empty(), "records for a small step");
+  if (tiles.empty()) return;
+  append_tiles_seen++;
+  std::size_t row = 0;
+  for (const TileRec& t : tiles) {
+    REQUIRE(t.row == (int)row && t.count >= 1 && t.slot >= 0 && t.slot + t.count <= kPageTokens,
+            "record at row %d: slot %d count %d", t.row, t.slot, t.count);
+    for (int i = 0; i < t.count; ++i, ++row) {
+      REQUIRE(row < st.rows.size(), "past the rows");
+      REQUIRE(st.rows[row].page == t.page && st.rows[row].slot == t.slot + i, "row %zu", row);
+    }
+  }
+  REQUIRE(row == st.rows.size(), "%zu of %zu rows", row, st.rows.size());
+}
+
 // The one-launch step lists: taken exactly when the step qualifies; each
 // (session, KV head) is one segment of at most kStepMaxParts pieces tiling
 // its pages in order; only the last piece appends and it holds every new
@@ -346,6 +370,7 @@ void random_plans(int cases) {
     for (int k = 0; k < ns; ++k) rows += d.n_new[(std::size_t)k];
     REQUIRE((int)st.rows.size() == rows, "rows");
     const bool i8 = rng() % 2, sf32 = rng() % 2;
+    check_append_tiles(st);
     check_step_lists(st, i8, sf32);
     {
       // the same sessions at head_dim 64, and a short slice of them (so
@@ -403,6 +428,7 @@ void random_plans(int cases) {
   REQUIRE(narrow_seen > 0 && wide_seen > 0, "tile widths: %d narrow, %d wide", narrow_seen,
           wide_seen);
   REQUIRE(appends_seen > 0, "no plan with new-row lists");
+  REQUIRE(append_tiles_seen > 0, "no plan with append page records");
 }
 
 void invalid_descriptions() {

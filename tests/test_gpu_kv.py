@@ -938,3 +938,34 @@ def test_random_append_bitexact(gpu, i):
     b.close()
     check_contents(case)
     case.close()
+
+
+@pytest.mark.parametrize("fmt,sf,kvh,hd", [
+    (tk.KV_F16, 0, 5, 100), (tk.KV_F16, 0, 4, 128), (tk.KV_F16, 0, 1, 256), (tk.KV_F16, 0, 2, 132),
+    (tk.KV_I8, 1, 5, 96), (tk.KV_I8, 0, 4, 128), (tk.KV_I8, 1, 2, 256), (tk.KV_I8, 0, 1, 224)])
+def test_append_whole_pages_bitexact(gpu, fmt, sf, kvh, hd):
+    """A step of many rows stores page by page: sessions that start at, after
+    and before a page edge, whole pages, pages shared with earlier rows and
+    a last wave that is not full; special values among them."""
+    case = PagedCase(kvh * 2, kvh, hd, fmt, [0, 16, 21, 500, 15], [1600, 1024, 1115, 533, 769],
+                     scale_format=sf, seed=31, outlier_frac=0.01 if fmt == tk.KV_I8 else 0)
+    rng = np.random.default_rng(5)
+    n = kvh * hd
+    for s, c in enumerate(case.contexts):
+        if fmt == tk.KV_F16:
+            for x in (case.k[s], case.v[s]):
+                for row in (c, c + 7, c + 60):
+                    x[row, rng.permutation(n)[:30]] = edge_values(30, rng)
+        for x in (case.k[s], case.v[s]):
+            x[c + 40, :32] = 0.0
+            x[c + 41, :32] = -0.0
+            x[c + 42, :32] *= np.float32(1e-30)
+    case.fill()
+    b = tk.Batch().plan(case.pool, case.sessions(True), case.qh)
+    dk, dv = (tk.DeviceArray.from_numpy(np.concatenate([a[c:] for a, c in zip(x, case.contexts)]))
+              for x in (case.k, case.v))
+    b.append(case.pool, 0, dk, dv)
+    tk.hip().sync()
+    b.close()
+    check_contents(case)
+    case.close()
