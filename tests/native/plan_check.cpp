@@ -431,6 +431,35 @@ void random_plans(int cases) {
   REQUIRE(append_tiles_seen > 0, "no plan with append page records");
 }
 
+// Block-prefill launches whose tiles do not come out at a multiple of the
+// compute units: the full rounds keep whole tiles and only the last,
+// partial round is cut (no piece below the smallest split); tiles that two
+// pieces fill one round with are not cut further.
+void prefill_rounds() {
+  struct {
+    int ctx, count, q_heads, kvh, hd, halves;
+    bool i8;
+    int pieces, parts;
+  } const cases[] = {{14003, 1333, 28, 4, 128, 2, true, 476, 220},
+                     {1536, 512, 16, 8, 256, 1, false, 256, 256}};
+  for (const auto& c : cases) {
+    std::vector<int> ids((std::size_t)(c.ctx + c.count + 15) / 16, 0);
+    const int off[2] = {0, (int)ids.size()};
+    Step st;
+    const char* msg = nullptr;
+    REQUIRE(build_step(st, 1, &c.ctx, &c.count, off, ids.data(), c.q_heads, c.kvh, c.hd, 1, &msg) == TGE_OK,
+            "%s", msg);
+    AttnLists pf;
+    build_prefill(st, 256, pf, 0, c.halves, c.i8);
+    check_lists(st, pf, 0, true);
+    REQUIRE((int)pf.work.size() == c.pieces && pf.parts == c.parts, "%zu pieces, %d parts", pf.work.size(),
+            pf.parts);
+    for (const WorkRec& w : pf.work)
+      REQUIRE(w.part < 0 || w.page_end - w.page_begin >= 32 * c.halves, "a piece of %d pages",
+              w.page_end - w.page_begin);
+  }
+}
+
 void invalid_descriptions() {
   const int ctx[2] = {20, 5}, nn[2] = {1, 2}, off[3] = {0, 2, 3}, ids[3] = {4, 5, 6};
   Step st;
@@ -497,6 +526,7 @@ void allocation_failures() {
 }
 
 int main() {
+  prefill_rounds();
   invalid_descriptions();
   allocation_failures();
   random_plans(600);
