@@ -36,12 +36,15 @@ __device__ __forceinline__ float pow2i(float e) {
   return __builtin_amdgcn_ldexpf(1.0f, (int)fmaxf(e, -300.0f));
 }
 
-// max(a, b, c) in one instruction (scores are never signalling NaNs, so
-// the operand quieting fmaxf would add is not needed).
+// max(a, b, c) ignoring NaN, one v_max3_f32 (maximumnum needs none of the
+// operand quieting that fmaxf adds). Not inline asm: the operands come
+// straight from MFMAs, whose results a vector instruction must not read for
+// several issue slots, and the compiler puts in those waits only before
+// instructions that it knows. (As inline asm the first two maxima after a
+// page pair's scores read two registers too early, so whether a row's base
+// moved at a page pair depended on timing.)
 __device__ __forceinline__ float max3f(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
+  return __builtin_elementwise_maximumnum(__builtin_elementwise_maximumnum(a, b), c);
 }
 
 template <typename T, typename F>

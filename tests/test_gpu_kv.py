@@ -428,6 +428,51 @@ def test_prefill_tile_widths(gpu, name):
     case.close()
 
 
+@pytest.mark.parametrize("qh,kvh,hd,contexts,n_new,kind", [
+    (28, 4, 128, [1500], [300], "prefill"), (16, 8, 128, [0], [1100], "prefill"), (14, 2, 64, [700], [400], "prefill"),
+    (16, 8, 256, [300], [200], "prefill"), (28, 4, 128, [900, 600], [4, 300], "mixed")])
+def test_prefill_rising_scores(gpu, qh, kvh, hd, contexts, n_new, kind):
+    """Every page pair holds one score 20 (log2) above all before it, at each
+    of a pair's positions in turn and all of it in the last 32 dims: a row
+    whose base did not follow it would overflow its f16 weights. The largest
+    weight of a row is 2^20 times the next, so its output is one V row."""
+    case = PagedCase(qh, kvh, hd, tk.KV_F16, contexts, n_new, seed=77, q_scale=0.05)
+    unit = 32 * math.log2(math.e) / math.sqrt(hd)  # log2 score of 1.0 in the last 32 dims
+    case.q.reshape(-1, hd)[:, hd - 32:] = 1.0
+    for k in case.k:
+        k *= np.float32(0.05)
+        pairs = -(-k.shape[0] // 32)
+        at = 32 * np.arange(pairs) + np.arange(pairs) * 7 % 32
+        at = at[at < k.shape[0]]
+        k.reshape(k.shape[0], kvh, hd)[at, :, hd - 32:] = (math.ceil(20 / unit) * np.arange(1, len(at) + 1))[:, None, None]
+    case.fill()
+    got, b = case.step(kind=kind)
+    assert np.isfinite(got).all()
+    assert_attention_close(got, case.oracle_out(), f"rising scores {kind}")
+    b.close()
+    case.close()
+
+
+@pytest.mark.parametrize("qh,kvh,hd,ctx,count", [(28, 4, 128, 1536, 512), (28, 4, 128, 0, 512), (16, 8, 128, 0, 1100),
+                                                 (14, 2, 64, 0, 777), (16, 8, 256, 512, 512)])
+def test_prefill_repeats_bit_for_bit(gpu, qh, kvh, hd, ctx, count):
+    """The same f16 chunk again gives the same bits: nothing in the kernel
+    depends on timing."""
+    case = PagedCase(qh, kvh, hd, tk.KV_F16, [ctx], [count], seed=78)
+    case.fill()
+    first, b = case.step(kind="prefill")
+    dq = tk.DeviceArray.from_numpy(case.q)
+    dout = tk.DeviceArray(case.q.shape, np.float32)
+    for i in range(30):
+        dout.zero()
+        b.prefill(case.pool, 0, dq, dout)
+        tk.hip().sync()
+        differ = int((dout.numpy().view(np.uint32) != first.view(np.uint32)).sum())
+        assert differ == 0, f"pass {i}: {differ} of {first.size} values differ"
+    b.close()
+    case.close()
+
+
 @pytest.mark.parametrize("fmt", [tk.KV_F16, tk.KV_I8])
 def test_pool_layer_beyond_4gib(gpu, fmt):
     """One layer's block array past 4 GiB: the kernels address each page

@@ -2,9 +2,12 @@
 on small hand-written listings: a register of an inline-asm ds_read_b64 that
 is copied, overwritten or used before the lgkmcnt(0) wait is reported; the
 same code with the wait first is clean. (The check itself runs over the
-real kernels with `make asm-check`.)"""
+real kernels with `make asm-check`.) And the sources' inline asm holds no
+vector ALU or matrix instruction."""
+import glob
 import importlib.util
 import os
+import re
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -65,3 +68,17 @@ def test_main_counts_kernels(tmp_path):
     assert m.main(str(f)) == 1
     f.write_text("\n".join(listing(READ + WAIT + "\tv_mov_b32_e32 v9, v64\n")) + "\n")
     assert m.main(str(f)) == 0
+
+
+def test_inline_asm_holds_no_vector_instruction():
+    """The compiler waits out an MFMA's result before vector instructions it
+    knows, not before one inside inline asm."""
+    seen = 0
+    for path in glob.glob(os.path.join(ROOT, "aegean-tge_amd", "csrc", "*")):
+        with open(path) as f:
+            text = f.read()
+        for m in re.finditer(r"\basm\b\s*(?:volatile\s*)?\(((?:\s*\"[^\"]*\")+)", text):
+            seen += 1
+            code = "".join(re.findall(r'"([^"]*)"', m.group(1)))
+            assert not re.search(r"\bv_\w+", code), f"{os.path.basename(path)}: {code}"
+    assert seen > 0
