@@ -317,39 +317,34 @@ void build_decode(const Step& b, Residency res, AttnLists& pl, int only) {
 
 namespace {
 
-// Splits [0, pages) into n nearly equal ranges (fewer if n does not divide
-// it) and appends one unit each.
+// Splits [0, pages) into n ranges that differ by at most a page and appends
+// one unit each.
 void add_units(std::vector<WorkRec>& work, std::vector<ReduceRec>& red, int& parts,
-               int& max_splits, WorkRec base, int pages, int n) {
-  n = std::min(n, pages);
-  if (n > 1) n = (pages + (pages + n - 1) / n - 1) / ((pages + n - 1) / n);
+               int& max_splits, WorkRec w, int pages, int n) {
   max_splits = std::max(max_splits, n);
+  w.part = w.red = -1;
   if (n == 1) {
-    base.page_begin = 0;
-    base.page_end = pages;
-    base.part = -1;
-    base.red = -1;
-    work.push_back(base);
+    w.page_begin = 0;
+    w.page_end = pages;
+    work.push_back(w);
     return;
   }
-  const int chunk = (pages + n - 1) / n;
   ReduceRec r{};
-  r.session = base.session;
-  r.row_begin = base.row_begin;
-  r.rows = base.rows;
-  r.rows_per_query = base.rows_per_query;
-  r.head_base = base.head_base;
+  r.session = w.session;
+  r.row_begin = w.row_begin;
+  r.rows = w.rows;
+  r.rows_per_query = w.rows_per_query;
+  r.head_base = w.head_base;
   r.first_part = parts;
-  r.q_row = base.q_row;
-  r.n_parts = 0;
-  for (int b = 0; b < pages; b += chunk) {
-    WorkRec w = base;
-    w.page_begin = b;
-    w.page_end = std::min(pages, b + chunk);
+  r.q_row = w.q_row;
+  r.n_parts = n;
+  w.red = (int)red.size();
+  w.page_end = 0;
+  for (int k = 0; k < n; ++k) {
+    w.page_begin = w.page_end;
+    w.page_end = (int)((long)pages * (k + 1) / n);
     w.part = parts++;
-    w.red = (int)red.size();
     work.push_back(w);
-    ++r.n_parts;
   }
   red.push_back(r);
 }
@@ -394,15 +389,13 @@ double launch_length(const std::vector<int>& lens, const std::vector<int>& cuts,
 // instead, where it is shorter by 3 %: every tile in as many pieces as one,
 // two or three rounds hold, or whole tiles for every full round with only the shortest tiles,
 // those of the last, partial round, cut so that they fill it (and few
-// partials to merge). Pieces keep at least min_pages pages. 256 CUs, before
-// and after: 300 tiles of 876 to 959 pages (int8, 128 dims) in 600 pieces,
+// partials to merge). No piece is shorter than half of min_pages. 256 CUs, before
+// and after: 300 tiles of 877 to 959 pages (int8, 128 dims) in 600 pieces,
 // three rounds for 2.3 rounds' work, or 256 whole tiles and 44 in 5 pieces:
 // 17.4 -> 14.3 ms over 28 layers; 128 tiles of 97 to 128 pages (f16, 256
 // dims) in 4 pieces each or in 2.
 void choose_cuts(const std::vector<int>& lens, int heads, int slots, int min_pages, std::vector<int>& cuts) {
   const long n = (long)lens.size() * heads;
-  long total = 0;
-  for (int l : lens) total += (long)l * heads;
   // (many rounds: the last one hardly counts)
   if (lens.empty() || n > 8L * slots) return;
   double best = 0.97 * launch_length(lens, cuts, heads, slots);

@@ -15,6 +15,7 @@
 // Prints "plan_check ok" and exits 0, or prints the first failure and
 // exits 1.
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -460,6 +461,43 @@ void prefill_rounds() {
   }
 }
 
+// Block-prefill launches of random prompts, at every block width and both
+// formats: pieces of a cut tile differ by at most a page and keep half of
+// the shortest length that is cut.
+void prefill_pieces(int cases) {
+  std::mt19937 rng(4242);
+  for (int i = 0; i < cases; ++i) {
+    const int hd = std::vector<int>{64, 96, 128, 256}[rng() % 4], kvh = 1 << (rng() % 4), group = 1 + (int)(rng() % 8);
+    const int ns = rng() % 4 ? 1 : 1 + (int)(rng() % 5), halves = hd > 64 && hd <= 128 ? 2 : 1;
+    std::vector<int> ctx, n, off{0}, ids;
+    for (int k = 0; k < ns; ++k) {
+      ctx.push_back((int)std::exp((double)(rng() % 1000) / 1000 * std::log(24000.0)) - 1);
+      n.push_back(65 + (int)(rng() % 3000));
+      ids.resize(ids.size() + (std::size_t)(ctx.back() + n.back() + 15) / 16, 0);
+      off.push_back((int)ids.size());
+    }
+    Step st;
+    const char* msg = nullptr;
+    REQUIRE(build_step(st, ns, ctx.data(), n.data(), off.data(), ids.data(), kvh * group, kvh, hd, 1, &msg) == TGE_OK,
+            "%s", msg);
+    AttnLists pf;
+    const bool i8 = rng() % 2;
+    build_prefill(st, 256, pf, 0, halves, i8);
+    check_lists(st, pf, 0, true);
+    std::map<int, std::pair<int, int>> span;  // merge record -> shortest and longest piece
+    for (const WorkRec& w : pf.work) {
+      const int len = w.page_end - w.page_begin;
+      if (w.red < 0) continue;
+      auto& s = span.emplace(w.red, std::make_pair(len, len)).first->second;
+      s = {std::min(s.first, len), std::max(s.second, len)};
+    }
+    for (const auto& s : span) {
+      REQUIRE(s.second.second - s.second.first <= 1, "pieces of %d to %d pages", s.second.first, s.second.second);
+      REQUIRE(s.second.first >= 16 * halves, "a piece of %d pages", s.second.first);
+    }
+  }
+}
+
 void invalid_descriptions() {
   const int ctx[2] = {20, 5}, nn[2] = {1, 2}, off[3] = {0, 2, 3}, ids[3] = {4, 5, 6};
   Step st;
@@ -527,6 +565,7 @@ void allocation_failures() {
 
 int main() {
   prefill_rounds();
+  prefill_pieces(1500);
   invalid_descriptions();
   allocation_failures();
   random_plans(600);
