@@ -4,7 +4,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <functional>
 
 #include "tge_kv.h"
 
@@ -353,78 +352,83 @@ void add_units(std::vector<WorkRec>& work, std::vector<ReduceRec>& red, int& par
 #define TGE_PREFILL_MIN_SPLIT 32
 #endif
 
-// Costs of a block-prefill launch beside its pages, in pages of one item:
-// an item's start and end, the merge launch, and one partial's way through
-// memory.
-constexpr double kPrefillItemCost = 16, kPrefillMergeCost = 18, kPrefillPartCost = 0.08;
+// What a block-prefill launch of its own costs on an MI355X, microseconds,
+// by kernel: the launch, an item's start and end, and a page of an item.
+// Where a compute unit holds three workgroups (64 dims), `page` is that of
+// an item alone there, and `two` and `three` times as much is a page of each
+// of two or three that share it. Fitted to 1,318 launches (12 to 1,500
+// items, 28/4, 12/2, 16/4 x 96, 14/2 x 64 and 16/8 x 256 heads, contexts up
+// to 24,000): 5 to 6 % rms off at 128 and 256 dims, 8 to 9 % at 64.
+struct PrefillCost {
+  double launch, item, page;
+  int per_cu;
+  double two, three;
+};
+PrefillCost prefill_cost(int block_dims, int tile_rows, bool i8) {
+  if (block_dims <= 64)
+    return i8 ? PrefillCost{8.0, 2.0, 0.327, 3, 1.57, 2.19} : PrefillCost{7.5, 2.9, 0.194, 3, 1.47, 2.17};
+  if (block_dims > 128) return i8 ? PrefillCost{3.0, 9.9, 0.899, 1, 1, 1} : PrefillCost{2.6, 9.6, 0.447, 1, 1, 1};
+  if (tile_rows == 64) return i8 ? PrefillCost{3.6, 6.1, 0.333, 1, 1, 1} : PrefillCost{3.3, 6.1, 0.167, 1, 1, 1};
+  return i8 ? PrefillCost{3.5, 9.9, 0.422, 1, 1, 1} : PrefillCost{3.2, 10.0, 0.230, 1, 1, 1};
+}
+// The merge launch behind it, and 64 KiB of partials through it (1,300
+// launches, 0.9 us rms off).
+constexpr double kMergeLaunch = 5.6, kMergePart = 0.0100;
 
-// Length of a launch whose tiles (`lens` pages each, once per KV head) are
-// cut into `cuts` pieces, in pages: the pieces go out longest first, each
-// to the first of `slots` workgroup slots that is free. One head's tiles on
-// its share of the slots stand for all.
-double launch_length(const std::vector<int>& lens, const std::vector<int>& cuts, int heads, int slots) {
-  std::vector<int> pieces;
-  long parts = 0;
-  for (std::size_t i = 0; i < lens.size(); ++i) {
-    const int len = (lens[i] + cuts[i] - 1) / cuts[i];
-    pieces.insert(pieces.end(), (std::size_t)cuts[i], len);
-    if (cuts[i] > 1) parts += cuts[i];
+// A way to cut a step's tiles: tiles of tile_rows rows (tq queries), of
+// lens[i] pages once per KV head, in cuts[i] pieces.
+struct TileCuts {
+  int tile_rows = 0, tq = 1;
+  std::vector<int> lens, cuts;
+};
+
+// The number of pieces of each length (0 to the longest) of one KV head.
+void piece_lengths(const TileCuts& c, std::vector<int>& count) {
+  int longest = 0;
+  for (std::size_t i = 0; i < c.lens.size(); ++i)
+    longest = std::max(longest, c.cuts[i] == 1 ? c.lens[i] : (c.lens[i] - 1) / c.cuts[i] + 1);
+  count.assign((std::size_t)longest + 1, 0);
+  for (std::size_t i = 0; i < c.lens.size(); ++i) {
+    if (c.cuts[i] == 1) {
+      count[(std::size_t)c.lens[i]]++;
+      continue;
+    }
+    const int len = c.lens[i] / c.cuts[i], more = c.lens[i] % c.cuts[i];
+    count[(std::size_t)len] += c.cuts[i] - more;
+    if (more) count[(std::size_t)len + 1] += more;
   }
-  std::sort(pieces.begin(), pieces.end(), std::greater<int>());
-  const std::size_t share = (std::size_t)std::max(1, slots / heads);
-  std::vector<double> busy(share, 0.0);  // a min-heap of the slots' ends
-  double end = 0.0;
-  for (std::size_t i = 0; i < pieces.size(); ++i) {
-    std::pop_heap(busy.begin(), busy.end(), std::greater<double>());
-    busy.back() += pieces[i] + kPrefillItemCost;
-    end = std::max(end, busy.back());
-    std::push_heap(busy.begin(), busy.end(), std::greater<double>());
-  }
-  return end + (parts ? kPrefillMergeCost + kPrefillPartCost * (double)parts * heads : 0.0);
 }
 
-// Cuts for a block-prefill launch of its own: `cuts` holds those of about
-// two rounds of equal pieces, which leave a last round nearly empty where
-// tiles times pieces does not come near a multiple of the slots. Taken
-// instead, where it is shorter by 3 %: every tile in as many pieces as one,
-// two or three rounds hold, or whole tiles for every full round with only the shortest tiles,
-// those of the last, partial round, cut so that they fill it (and few
-// partials to merge). No piece is shorter than half of min_pages. 256 CUs, before
-// and after: 300 tiles of 877 to 959 pages (int8, 128 dims) in 600 pieces,
-// three rounds for 2.3 rounds' work, or 256 whole tiles and 44 in 5 pieces:
-// 17.4 -> 14.3 ms over 28 layers; 128 tiles of 97 to 128 pages (f16, 256
-// dims) in 4 pieces each or in 2.
-void choose_cuts(const std::vector<int>& lens, int heads, int slots, int min_pages, std::vector<int>& cuts) {
-  const long n = (long)lens.size() * heads;
-  // (many rounds: the last one hardly counts)
-  if (lens.empty() || n > 8L * slots) return;
-  double best = 0.97 * launch_length(lens, cuts, heads, slots);
-  const auto take = [&](const std::vector<int>& c) {
-    const double t = launch_length(lens, c, heads, slots);
-    if (t < best) {
-      best = t;
-      cuts = c;
+// Microseconds of the launch that `c` gives. The pieces go out longest
+// first: with L(i) the length of the i-th and S workgroups at once, the end
+// is past k + 1 pieces of length L(k * S) for every k, and past all pages
+// divided by S. (`count`: scratch.)
+double launch_time(const TileCuts& c, const PrefillCost& cost, int heads, int cus, int block_dims,
+                   std::vector<int>& count) {
+  piece_lengths(c, count);
+  const long slots = (long)cus * cost.per_cu;
+  long rank = 0, next = 0, round = 0, pages = 0, parts = 0;
+  double t = 0.0, shared[3] = {0, 0, 0};
+  for (int len = (int)count.size() - 1; len > 0; --len) {
+    if (!count[(std::size_t)len]) continue;
+    const long n = (long)count[(std::size_t)len] * heads;
+    rank += n;
+    pages += n * len;
+    for (; next < rank; next += cus, ++round) {
+      if (cost.per_cu == 1)
+        t = std::max(t, (double)(round + 1) * (cost.item + cost.page * len));
+      else if (round < 3)
+        shared[round] = len;
     }
-  };
-  std::vector<int> c(lens.size());
-  for (int rounds : {1, 2, 3}) {
-    const int pieces = (int)std::max<long>(1, rounds * (long)slots / n);
-    for (std::size_t i = 0; i < lens.size(); ++i) c[i] = std::max(1, std::min(pieces, lens[i] / min_pages));
-    take(c);
   }
-  const long rest = n % slots;
-  if (rest == 0 || rest == n) return;
-  std::vector<std::size_t> order(lens.size());
-  for (std::size_t i = 0; i < order.size(); ++i) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](std::size_t x, std::size_t y) { return lens[x] < lens[y]; });
-  const std::size_t tail = (std::size_t)((rest + heads - 1) / heads);  // tiles of one head
-  const int most = (int)std::max<long>(1, slots / ((long)tail * heads));
-  for (int pieces : {most, most + 1}) {
-    std::fill(c.begin(), c.end(), 1);
-    for (std::size_t k = 0; k < tail; ++k)
-      c[order[k]] = std::max(1, std::min(pieces, lens[order[k]] / min_pages));
-    take(c);
-  }
+  if (cost.per_cu > 1)  // the first compute unit's: three, then two, then one at work
+    t = cost.item + cost.page * (shared[2] * cost.three + (shared[1] - shared[2]) * cost.two + (shared[0] - shared[1]));
+  if (rank > slots)
+    t = std::max(t, (cost.page * (double)pages + cost.item * (double)rank) * cost.three / (double)slots);
+  for (int cuts : c.cuts) parts += cuts > 1 ? cuts : 0;
+  if (parts)
+    t += kMergeLaunch + kMergePart * (double)(parts * heads) * prefill_tile_rows(block_dims) * block_dims / 16384.0;
+  return cost.launch + t;
 }
 
 }  // namespace
@@ -436,74 +440,86 @@ void build_prefill(const Step& b, int cus, AttnLists& pl, int only, int halves, 
   pl.groups = 0;
   pl.parts = pl.max_splits = 0;
   pl.row_groups = kPrefillRows / 16;
+  cus = std::max(1, cus);
   halves = halves == 2 ? 2 : 1;
-  // Page-split size for tiles of tq queries: enough items for about two
+  const int min_pages = TGE_PREFILL_MIN_SPLIT * halves;
+  // Tiles of tile_rows rows in pieces of about equal length: enough for two
   // rounds of two four-wave workgroups on each compute unit (of one
-  // eight-wave workgroup with two halves), at least 32 pages (eight tiles
-  // of four) per half. `pieces` counts the workgroups that gives.
-  const long target_units = 2L * std::max(1, cus) * (halves == 2 ? 1 : 2);
-  auto split_size = [&](int tq, long* pieces) {
-    long pages_total = 0;
+  // eight-wave workgroup with two halves). A tile is cut when it is longer
+  // than min_pages.
+  const auto equal_pieces = [&](int tile_rows) {
+    TileCuts c;
+    c.tile_rows = tile_rows;
+    c.tq = std::max(1, tile_rows / b.group);
+    long total = 0;
     for (const auto& sr : b.sessions) {
       if (!take_session(b, sr, only)) continue;
-      for (int a = 0; a < sr.n_new; a += tq)
-        pages_total += (long)((sr.ctx + std::min(sr.n_new, a + tq) + 15) / 16) * b.kv_heads;
-    }
-    const int pps = (int)std::max<long>((long)TGE_PREFILL_MIN_SPLIT * halves,
-                                        ((pages_total + target_units - 1) / target_units + 3) / 4 * 4);
-    if (pieces) {
-      *pieces = 0;
-      for (const auto& sr : b.sessions) {
-        if (!take_session(b, sr, only)) continue;
-        for (int a = 0; a < sr.n_new; a += tq)
-          *pieces += (long)(((sr.ctx + std::min(sr.n_new, a + tq) + 15) / 16 + pps - 1) / pps) *
-                     b.kv_heads;
+      for (int a = 0; a < sr.n_new; a += c.tq) {
+        c.lens.push_back((sr.ctx + a + std::min(c.tq, sr.n_new - a) + 15) / 16);
+        total += (long)c.lens.back() * b.kv_heads;
       }
     }
-    return pps;
+    const long units = 2L * cus * (halves == 2 ? 1 : 2);
+    const int pps = (int)std::max<long>(min_pages, ((total + units - 1) / units + 3) / 4 * 4);
+    c.cuts.resize(c.lens.size());
+    for (std::size_t i = 0; i < c.lens.size(); ++i)
+      c.cuts[i] = (c.lens[i] + pps - 1) / pps;
+    return c;
   };
-  pl.tile_rows = prefill_tile_rows(b.block_dims);
-  int tq = std::max(1, pl.tile_rows / b.group);
-  int pps = split_size(tq, nullptr);
-  // Narrow tiles: a 128-dim step whose 128-row tiles would leave half the
-  // compute units idle (the two-halves kernel runs one workgroup per CU)
-  // takes 64-row tiles (one 16-row group per wave) instead: twice the
-  // workgroups, each with half the rows against the same pages. With f16
-  // pages, so does a step whose 128-row tiles would be split and merged
-  // while its 64-row tiles fit one round of workgroups unsplit.
-  if (halves == 2 && b.block_dims == 128 && b.group <= 64) {
-    long pieces = 0, items = 0;
-    split_size(tq, &pieces);
-    const int tq64 = std::max(1, 64 / b.group);
-    for (const auto& sr : b.sessions)
-      if (take_session(b, sr, only)) items += (long)((sr.n_new + tq64 - 1) / tq64) * b.kv_heads;
-    if (2 * pieces <= std::max(1, cus)) {
-      pl.tile_rows = 64;
-      tq = tq64;
-      pps = split_size(tq, nullptr);
-    } else if (!i8 && items <= std::max(1, cus) && pieces > items / 2) {
-      // the split 128-row tiles need a merge launch; one round of unsplit
-      // 64-row tiles does not (f16 pages: with int8 ones the split
-      // 128-row tiles measure faster)
-      pl.tile_rows = 64;
-      tq = tq64;
-      pps = 1 << 30;
+  TileCuts best = equal_pieces(prefill_tile_rows(b.block_dims));
+  std::vector<int> count;
+  // A launch of its own takes the shortest of a few ways: those pieces, whole
+  // tiles, every tile in as many pieces as one, two or three rounds hold, or
+  // whole tiles for the full rounds and only the shortest, those of the
+  // last, partial round, in pieces that fill it; at 128 dims with two halves
+  // each of these for 128-row tiles and for 64-row ones (one 16-row group
+  // per wave), whose items are twice as many and cost less than half as
+  // much more a page. Ways with a merge launch have to be 5 % shorter than
+  // whole tiles. No piece is shorter than half of min_pages. (Tiles beside a
+  // decode role, or in two workgroups of 128 dims per unit, keep equal
+  // pieces: neither has been fitted.)
+  if (only == 0 && !best.lens.empty() && (halves == 2 || b.block_dims != 128)) {
+    double best_time = 1e30;
+    const int widths = b.block_dims == 128 && b.group <= 64 ? 2 : 1;
+    TileCuts ways[2] = {std::move(best), widths > 1 ? equal_pieces(64) : TileCuts{}};
+    for (int w = 0; w < widths; ++w) {
+      TileCuts& c = ways[w];
+      const PrefillCost cost = prefill_cost(b.block_dims, c.tile_rows, i8);
+      const long n = (long)c.lens.size() * b.kv_heads, slots = (long)cus * cost.per_cu;
+      const auto take = [&] {
+        const bool whole = std::all_of(c.cuts.begin(), c.cuts.end(), [](int x) { return x == 1; });
+        const double t = launch_time(c, cost, b.kv_heads, cus, b.block_dims, count) * (whole ? 0.95 : 1.0);
+        if (t >= best_time) return;
+        best_time = t;
+        best = c;
+      };
+      take();
+      long last = 0;
+      for (long pieces : {1L, slots / n, 2 * slots / n, 3 * slots / n}) {
+        if (pieces <= last) continue;
+        last = pieces;
+        for (std::size_t i = 0; i < c.lens.size(); ++i)
+          c.cuts[i] = (int)std::max<long>(1, std::min<long>(pieces, c.lens[i] / min_pages));
+        take();
+      }
+      const long rest = n % slots;
+      if (n < slots || rest == 0) continue;
+      std::vector<std::size_t> order(c.lens.size());
+      for (std::size_t i = 0; i < order.size(); ++i) order[i] = i;
+      const std::size_t tail = (std::size_t)((rest + b.kv_heads - 1) / b.kv_heads);  // tiles of one head
+      std::nth_element(order.begin(), order.begin() + (std::ptrdiff_t)tail - 1, order.end(),
+                       [&](std::size_t x, std::size_t y) { return c.lens[x] != c.lens[y] ? c.lens[x] < c.lens[y] : x < y; });
+      const long most = slots / ((long)tail * b.kv_heads);
+      for (long pieces : {most, most + 1}) {
+        if (pieces < 2) continue;
+        std::fill(c.cuts.begin(), c.cuts.end(), 1);
+        for (std::size_t k = 0; k < tail; ++k)
+          c.cuts[order[k]] = (int)std::max<long>(1, std::min<long>(pieces, c.lens[order[k]] / min_pages));
+        take();
+      }
     }
   }
-  // Pages per tile of one KV head (every head has the same tiles), and how
-  // many pieces each tile is cut into.
-  std::vector<int> lens;
-  for (const auto& sr : b.sessions) {
-    if (!take_session(b, sr, only)) continue;
-    for (int a = 0; a < sr.n_new; a += tq)
-      lens.push_back((sr.ctx + a + std::min(tq, sr.n_new - a) + 15) / 16);
-  }
-  std::vector<int> cuts(lens.size());
-  for (std::size_t i = 0; i < lens.size(); ++i) cuts[i] = std::max(1, (lens[i] + pps - 1) / pps);
-  if (only == 0 && pps < (1 << 30)) {
-    const int slots = std::max(1, cus) * (halves == 2 || b.block_dims > 128 ? 1 : 2);
-    choose_cuts(lens, b.kv_heads, slots, TGE_PREFILL_MIN_SPLIT * halves, cuts);
-  }
+  pl.tile_rows = best.tile_rows;
   std::size_t tile = 0;
   for (int s = 0; s < (int)b.sessions.size(); ++s) {
     const SessionRec& sr = b.sessions[(std::size_t)s];
@@ -511,7 +527,7 @@ void build_prefill(const Step& b, int cus, AttnLists& pl, int only, int halves, 
     const std::size_t tile0 = tile;
     for (int h = 0; h < b.kv_heads; ++h) {
       tile = tile0;
-      for (int a = 0; a < sr.n_new; a += tq, ++tile) {
+      for (int a = 0; a < sr.n_new; a += best.tq, ++tile) {
         WorkRec w{};
         w.session = s;
         w.kv_head = h;
@@ -519,10 +535,10 @@ void build_prefill(const Step& b, int cus, AttnLists& pl, int only, int halves, 
         w.q_row = sr.q_row;
         w.table_off = sr.table_off;
         w.row_begin = a;
-        w.rows = std::min(tq, sr.n_new - a) * b.group;
+        w.rows = std::min(best.tq, sr.n_new - a) * b.group;
         w.rows_per_query = b.group;
         w.head_base = h * b.group;
-        add_units(pl.work, pl.reduce, pl.parts, pl.max_splits, w, lens[tile], cuts[tile]);
+        add_units(pl.work, pl.reduce, pl.parts, pl.max_splits, w, best.lens[tile], best.cuts[tile]);
       }
     }
   }

@@ -141,14 +141,13 @@ void build_decode(const Step& s, Residency res, AttnLists& out, int only);
 // (app_waves 0) when `waves` is 0 or a wave would hold more than max_rows.
 void build_decode_appends(const Step& s, AttnLists& pl, int waves, int max_rows);
 
-// Block-prefill work: (session, KV head, query tile) x page splits sized so
-// the launch covers `cus` compute units about twice; longest items first.
-// `halves`: groups of four waves per workgroup (2: an item's pages are
-// shared by two halves, so items may be twice as long). At 128 dims with
-// two halves the tiles may be 64 rows (tile_rows) when 128-row tiles would
-// leave compute units idle; `i8`: int8 pages (whose dequantisation makes a
-// page read serve fewer rows at a higher cost, so unsplit 64-row tiles do
-// not replace split 128-row ones).
+// Block-prefill work: (session, KV head, query tile) x page pieces, longest
+// items first. `halves`: groups of four waves per workgroup (2: an item's
+// pages are shared by two halves). A launch of its own (`only` 0) takes the
+// shortest of a few ways to cut the tiles, by a model of the launch's length
+// on `cus` compute units (`i8`: int8 pages); at 128 dims with two halves the
+// tiles may be 64 rows (tile_rows). Otherwise the pieces are of about equal
+// length and cover the compute units about twice.
 void build_prefill(const Step& s, int cus, AttnLists& out, int only, int halves = 1,
                    bool i8 = false);
 

@@ -9,6 +9,28 @@ import oracle as O
 import synth
 import tge_kv as tk
 
+# Block prefills of one session by what their launch is made of on 256 compute
+# units (checked against the planner by test_host_plan.py, run by
+# test_gpu_kv.py): "whole" tiles, "cut" ones with a merge launch, or a "mix".
+# name: (q_heads, kv_heads, head_dim, format, context, rows, kind, tile rows)
+PREFILL_PLANS = {
+    "mix_128_f16": (64, 8, 128, tk.KV_F16, 3100, 560, "mix", 128),
+    "mix_128_i8": (64, 8, 128, tk.KV_I8, 3100, 560, "mix", 128),
+    "mix_256_f16": (16, 8, 256, tk.KV_F16, 1100, 1056, "mix", 64),
+    "mix_256_i8": (16, 8, 256, tk.KV_I8, 1100, 1056, "mix", 64),
+    "whole_128_f16": (28, 4, 128, tk.KV_F16, 0, 1333, "whole", 128),
+    "whole_128_i8": (28, 4, 128, tk.KV_I8, 0, 1333, "whole", 128),
+    "cut_64_f16": (14, 2, 64, tk.KV_F16, 1500, 900, "cut", 128),
+    "cut_64_i8": (14, 2, 64, tk.KV_I8, 1500, 900, "cut", 128),
+    "cut_96_narrow_i8": (16, 4, 96, tk.KV_I8, 1536, 512, "cut", 64),
+}
+# Steps whose append goes page by page, and the (format, scale format, KV
+# heads, head_dim) they are run at.
+PAGE_APPEND_STEP = ([0, 16, 21, 500, 15], [1600, 1024, 1115, 533, 769])
+PAGE_APPENDS = [
+    (tk.KV_F16, 0, 5, 100), (tk.KV_F16, 0, 4, 128), (tk.KV_F16, 0, 1, 256), (tk.KV_F16, 0, 2, 132),
+    (tk.KV_I8, 1, 5, 96), (tk.KV_I8, 0, 4, 128), (tk.KV_I8, 1, 2, 256), (tk.KV_I8, 0, 1, 224)]
+
 
 class PagedCase:
     def __init__(self, q_heads, kv_heads, head_dim, fmt, contexts, n_new, scale_format=0,

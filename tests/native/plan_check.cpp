@@ -498,6 +498,27 @@ void prefill_pieces(int cases) {
   }
 }
 
+// Launches that were once cut into too few pieces, int8 (measured,
+// microseconds, then / with at least `pieces`): 16/8 heads of 256 dims, 256
+// rows at context 512 (52 / 42) and 512 rows at 384 (59 / 50); 14/2 heads of
+// 64 dims, 2048 rows at 6000 (135 / 128) and at 8000 (164 / 150).
+void prefill_cut_where_faster() {
+  const struct {
+    int ctx, count, q_heads, kvh, hd, pieces;
+  } cases[] = {{512, 256, 16, 8, 256, 128}, {384, 512, 16, 8, 256, 200}, {6000, 2048, 14, 2, 64, 2 * 456},
+               {8000, 2048, 14, 2, 64, 2 * 456}};
+  for (const auto& c : cases) {
+    std::vector<int> ids((std::size_t)(c.ctx + c.count + 15) / 16, 0);
+    const int off[2] = {0, (int)ids.size()};
+    Step st;
+    const char* msg = nullptr;
+    REQUIRE(build_step(st, 1, &c.ctx, &c.count, off, ids.data(), c.q_heads, c.kvh, c.hd, 1, &msg) == TGE_OK, "%s", msg);
+    AttnLists pf;
+    build_prefill(st, 256, pf, 0, 1, true);
+    REQUIRE((int)pf.work.size() >= c.pieces, "%d rows at %d: %zu pieces", c.count, c.ctx, pf.work.size());
+  }
+}
+
 void invalid_descriptions() {
   const int ctx[2] = {20, 5}, nn[2] = {1, 2}, off[3] = {0, 2, 3}, ids[3] = {4, 5, 6};
   Step st;
@@ -563,9 +584,38 @@ void allocation_failures() {
   REQUIRE(m.live == 0, "leaked");
 }
 
-int main() {
+// plan_check <q_heads> <kv_heads> <head_dim> <int8> <ctx> <n_new> [<ctx>
+// <n_new> ...]: prints what the planner does with the step on 256 compute
+// units (items and partials of its block prefill, page records of its append).
+int describe(int argc, char** argv) {
+  std::vector<int> a;
+  for (int i = 1; i < argc; ++i) a.push_back(std::atoi(argv[i]));
+  if (a.size() < 6 || a.size() % 2) return 2;
+  std::vector<int> ctx, n, off{0}, ids;
+  for (std::size_t i = 4; i < a.size(); i += 2) {
+    ctx.push_back(a[i]);
+    n.push_back(a[i + 1]);
+    ids.resize(ids.size() + (std::size_t)(a[i] + a[i + 1] + 15) / 16, 0);
+    off.push_back((int)ids.size());
+  }
+  Step st;
+  const char* msg = nullptr;
+  if (build_step(st, (int)n.size(), ctx.data(), n.data(), off.data(), ids.data(), a[0], a[1], a[2], 1, &msg) != TGE_OK)
+    return 2;
+  AttnLists pf;
+  build_prefill(st, 256, pf, 0, st.block_dims == 128 ? 2 : 1, a[3] != 0);
+  std::vector<TileRec> tiles;
+  build_append_tiles(st, tiles);
+  std::printf("items %zu parts %d tile_rows %d append_pages %zu\n", pf.work.size(), pf.parts, pf.tile_rows,
+              tiles.size());
+  return 0;
+}
+
+int main(int argc, char** argv) {
+  if (argc > 1) return describe(argc, argv);
   prefill_rounds();
   prefill_pieces(1500);
+  prefill_cut_where_faster();
   invalid_descriptions();
   allocation_failures();
   random_plans(600);

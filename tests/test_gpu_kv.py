@@ -9,7 +9,7 @@ import pytest
 import oracle as O
 import synth
 import tge_kv as tk
-from _paged import PagedCase
+from _paged import PAGE_APPEND_STEP, PAGE_APPENDS, PREFILL_PLANS, PagedCase
 from _util import assert_attention_close, bits
 
 pytestmark = pytest.mark.gpu
@@ -396,11 +396,11 @@ def test_prefill_chunks_match_oracle(gpu):
 
 
 # Block prefill at head_dim 128 in both tile widths: (q_heads, kv_heads,
-# format, contexts, n_new). On 256 compute units the planner takes 128-row
-# tiles for the "wide" cases (144 items; 280 as 64-row tiles), unsplit
-# 64-row tiles where the 128-row ones would be split and merged (136
-# pieces of 68 tiles; 136 narrow items; f16 only: int8 keeps the split
-# 128-row tiles) and 64-row tiles for a small step (56 items).
+# format, contexts, n_new). On 256 compute units the planner takes 280
+# unsplit 64-row tiles for the first two, 136 unsplit 64-row tiles (f16) or
+# 68 128-row tiles in two pieces each (int8) for the next, and 56 64-row
+# tiles for the small step. (PREFILL_PLANS has launches of whole 128-row
+# tiles.)
 TILE_CASES = {
     "wide_f16": (16, 8, tk.KV_F16, [0], [1100]),
     "wide_i8": (16, 8, tk.KV_I8, [0], [1100]),
@@ -425,6 +425,25 @@ def test_prefill_tile_widths(gpu, name):
     assert tk.wait_expiries() == 0, "a bounded in-kernel wait ran out"
     b.close()
     check_contents(case)
+    case.close()
+
+
+@pytest.mark.parametrize("name", list(PREFILL_PLANS))
+def test_prefill_whole_and_cut_tiles(gpu, name):
+    """Launches of whole tiles, of cut ones with their merge and of both
+    (test_host_plan.py holds the plans to that): the first and the last query
+    of every tile against the oracle."""
+    qh, kvh, hd, fmt, ctx, n, _, tile_rows = PREFILL_PLANS[name]
+    case = PagedCase(qh, kvh, hd, fmt, [ctx], [n], seed=91, outlier_frac=0.01 if fmt == tk.KV_I8 else 0)
+    case.fill()
+    got, b = case.step(kind="prefill")
+    b.close()
+    fc = case.flat(0)
+    tq = tile_rows // (qh // kvh)
+    rows = sorted({r for a in range(0, n, tq) for r in (a, min(a + tq, n) - 1)})
+    want = np.concatenate([fc.attend(case.q[r:r + 1], qh, kvh, hd, ctx + r) for r in rows])
+    err = assert_attention_close(got[rows], want, f"prefill {name}")
+    say(f"  {len(rows)} rows, max abs err {err:.2e}")
     case.close()
 
 
@@ -985,15 +1004,13 @@ def test_random_append_bitexact(gpu, i):
     case.close()
 
 
-@pytest.mark.parametrize("fmt,sf,kvh,hd", [
-    (tk.KV_F16, 0, 5, 100), (tk.KV_F16, 0, 4, 128), (tk.KV_F16, 0, 1, 256), (tk.KV_F16, 0, 2, 132),
-    (tk.KV_I8, 1, 5, 96), (tk.KV_I8, 0, 4, 128), (tk.KV_I8, 1, 2, 256), (tk.KV_I8, 0, 1, 224)])
+@pytest.mark.parametrize("fmt,sf,kvh,hd", PAGE_APPENDS)
 def test_append_whole_pages_bitexact(gpu, fmt, sf, kvh, hd):
     """A step of many rows stores page by page: sessions that start at, after
     and before a page edge, whole pages, pages shared with earlier rows and
     a last wave that is not full; special values among them."""
-    case = PagedCase(kvh * 2, kvh, hd, fmt, [0, 16, 21, 500, 15], [1600, 1024, 1115, 533, 769],
-                     scale_format=sf, seed=31, outlier_frac=0.01 if fmt == tk.KV_I8 else 0)
+    case = PagedCase(kvh * 2, kvh, hd, fmt, *PAGE_APPEND_STEP, scale_format=sf, seed=31,
+                     outlier_frac=0.01 if fmt == tk.KV_I8 else 0)
     rng = np.random.default_rng(5)
     n = kvh * hd
     for s, c in enumerate(case.contexts):
@@ -1005,6 +1022,8 @@ def test_append_whole_pages_bitexact(gpu, fmt, sf, kvh, hd):
             x[c + 40, :32] = 0.0
             x[c + 41, :32] = -0.0
             x[c + 42, :32] *= np.float32(1e-30)
+            if fmt == tk.KV_I8:  # a whole page holds these rows, and a shared one the first
+                x[c + 43, 5], x[c + 44, 40], x[c, 7] = np.inf, np.nan, -np.inf
     case.fill()
     b = tk.Batch().plan(case.pool, case.sessions(True), case.qh)
     dk, dv = (tk.DeviceArray.from_numpy(np.concatenate([a[c:] for a, c in zip(x, case.contexts)]))

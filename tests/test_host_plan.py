@@ -22,7 +22,7 @@ FLAGS = ["-std=c++20", "-O1", "-g", "-fsanitize=address,undefined",
          "-I" + os.path.join(ROOT, "include")]
 
 
-def build_and_run(tmp_path, name, sources):
+def build_and_run(tmp_path, name, sources, runs=((),)):
     if not shutil.which("g++"):
         pytest.skip("g++ not available")
     exe = str(tmp_path / name)
@@ -31,9 +31,12 @@ def build_and_run(tmp_path, name, sources):
     assert r.returncode == 0, r.stderr[-4000:]
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1:abort_on_error=0",
                UBSAN_OPTIONS="print_stacktrace=1")
-    r = subprocess.run([exe], capture_output=True, text=True, timeout=300, env=env)
-    assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
-    return r.stdout
+    out = ""
+    for args in runs:
+        r = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=300, env=env)
+        assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
+        out += r.stdout
+    return out
 
 
 def test_planner_under_sanitizers(tmp_path):
@@ -46,3 +49,19 @@ def test_driver_bookkeeping_under_sanitizers(tmp_path):
     out = build_and_run(tmp_path, "driver_host_check",
                         ["aegean-tge_amd/host/qwen2_kv.cpp", "tests/native/driver_host_check.cpp"])
     assert "driver_host_check ok" in out
+
+
+def test_plans_of_the_gpu_cases(tmp_path):
+    """The GPU tests' launches are what they are named for."""
+    from _paged import PAGE_APPEND_STEP, PAGE_APPENDS, PREFILL_PLANS
+    import tge_kv as tk
+    runs = [(qh, kvh, hd, int(fmt == tk.KV_I8), ctx, n) for qh, kvh, hd, fmt, ctx, n, _, _ in PREFILL_PLANS.values()]
+    steps = [x for pair in zip(*PAGE_APPEND_STEP) for x in pair]
+    runs += [(2 * kvh, kvh, hd, int(fmt == tk.KV_I8), *steps) for fmt, _, kvh, hd in PAGE_APPENDS]
+    out = build_and_run(tmp_path, "plan_check", ["aegean-tge_amd/host/plan.cpp", "tests/native/plan_check.cpp"], runs)
+    plans = [dict(zip(line.split()[::2], map(int, line.split()[1::2]))) for line in out.splitlines()]
+    for (name, case), p in zip(PREFILL_PLANS.items(), plans):
+        kind = "whole" if p["parts"] == 0 else "cut" if p["parts"] == p["items"] else "mix"
+        assert (kind, p["tile_rows"]) == case[6:], (name, p)
+    for case, p in zip(PAGE_APPENDS, plans[len(PREFILL_PLANS):]):
+        assert p["append_pages"] > 0, case
