@@ -316,16 +316,16 @@ void build_decode(const Step& b, Residency res, AttnLists& pl, int only) {
 
 namespace {
 
-// Splits [0, pages) into n ranges that differ by at most a page and appends
-// one unit each.
-void add_units(std::vector<WorkRec>& work, std::vector<ReduceRec>& red, int& parts,
+// Splits [0, pages) into n ranges that differ by at most a page, one unit
+// each; a unit of len pages goes to work[at[len]++].
+void add_units(std::vector<WorkRec>& work, std::vector<int>& at, std::vector<ReduceRec>& red, int& parts,
                int& max_splits, WorkRec w, int pages, int n) {
   max_splits = std::max(max_splits, n);
   w.part = w.red = -1;
   if (n == 1) {
     w.page_begin = 0;
     w.page_end = pages;
-    work.push_back(w);
+    work[(std::size_t)at[(std::size_t)pages]++] = w;
     return;
   }
   ReduceRec r{};
@@ -343,7 +343,7 @@ void add_units(std::vector<WorkRec>& work, std::vector<ReduceRec>& red, int& par
     w.page_begin = w.page_end;
     w.page_end = (int)((long)pages * (k + 1) / n);
     w.part = parts++;
-    work.push_back(w);
+    work[(std::size_t)at[(std::size_t)(w.page_end - w.page_begin)]++] = w;
   }
   red.push_back(r);
 }
@@ -520,6 +520,16 @@ void build_prefill(const Step& b, int cus, AttnLists& pl, int only, int halves, 
     }
   }
   pl.tile_rows = best.tile_rows;
+  // Longest items first (partial slots are fixed per item, so order is free):
+  // the place of the first item of each length.
+  piece_lengths(best, count);
+  int items = 0;
+  for (std::size_t len = count.size(); len-- > 0;) {
+    const int n = count[len] * b.kv_heads;
+    count[len] = items;
+    items += n;
+  }
+  pl.work.resize((std::size_t)items);
   std::size_t tile = 0;
   for (int s = 0; s < (int)b.sessions.size(); ++s) {
     const SessionRec& sr = b.sessions[(std::size_t)s];
@@ -538,14 +548,10 @@ void build_prefill(const Step& b, int cus, AttnLists& pl, int only, int halves, 
         w.rows = std::min(best.tq, sr.n_new - a) * b.group;
         w.rows_per_query = b.group;
         w.head_base = h * b.group;
-        add_units(pl.work, pl.reduce, pl.parts, pl.max_splits, w, best.lens[tile], best.cuts[tile]);
+        add_units(pl.work, count, pl.reduce, pl.parts, pl.max_splits, w, best.lens[tile], best.cuts[tile]);
       }
     }
   }
-  // Longest items first (partial slots are fixed per item, so order is free).
-  std::stable_sort(pl.work.begin(), pl.work.end(), [](const WorkRec& x, const WorkRec& y) {
-    return x.page_end - x.page_begin > y.page_end - y.page_begin;
-  });
   pl.groups = (int)pl.work.size();
 }
 
