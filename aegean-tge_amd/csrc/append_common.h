@@ -30,21 +30,14 @@ template <int FMT>
 __device__ __forceinline__ LaneCodes encode_lane(const float (&x)[8]) {
   LaneCodes c{{0, 0, 0, 0}, 0.0f};
   if (FMT == kF16) {
-    // Normal halves need no branch: with t = |x|'s bits, the kept mantissa
-    // plus the guard bit is (t + 2^12) >> 13, less the exponents' offset.
-    // A lane with any other value (below 2^-14, past the f16 range, not
-    // finite) takes the recipe for all eight.
+    // Normal halves need no branch; a lane with any other value takes the
+    // recipe for all eight.
     bool normal = true;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      normal = normal && (f32_as_u32(x[i]) & 0x7fffffffu) - 0x38800000u < 0x0f000000u;
+    for (int i = 0; i < 8; ++i) normal = normal && half_is_normal(x[i]);
     if (normal) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t u = f32_as_u32(x[i]);
-        const uint32_t h = ((((u & 0x7fffffffu) + 0x1000u) >> 13) - 0x1c000u) | ((u >> 16) & 0x8000u);
-        c.w[i >> 1] |= h << (16 * (i & 1));
-      }
+      for (int i = 0; i < 8; ++i) c.w[i >> 1] |= (uint32_t)normal_to_half(x[i]) << (16 * (i & 1));
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i)

@@ -121,6 +121,18 @@ __host__ __device__ inline uint16_t float_to_half_ref(float value) {
   return (uint16_t)(sign | (kept + ((frac >> 12) & 1u)));
 }
 
+// The recipe without a branch for magnitudes from 2^-14 up to 65536: with t
+// the magnitude's bits, the kept mantissa plus the guard bit is
+// (t + 2^12) >> 13, less the exponents' offset (a carry out of the largest
+// half gives infinity, as the recipe does).
+__host__ __device__ inline bool half_is_normal(float value) {
+  return (f32_as_u32(value) & 0x7FFFFFFFu) - 0x38800000u < 0x0F000000u;
+}
+__host__ __device__ inline uint32_t normal_to_half(float value) {
+  const uint32_t u = f32_as_u32(value);
+  return ((((u & 0x7FFFFFFFu) + 0x1000u) >> 13) - 0x1C000u) | ((u >> 16) & 0x8000u);
+}
+
 // static_cast<int>(float) as the reference's x86-64 build executes it
 // (cvttss2si): truncation toward zero, INT_MIN for NaN and out-of-range.
 __host__ __device__ inline int trunc_to_int_x86(float r) {

@@ -453,6 +453,28 @@ def test_split_absmax_fold_matches_sequential():
         shutil.rmtree(d, ignore_errors=True)
 
 
+def test_normal_half_path_matches_recipe():
+    """The append's branch-free f16 conversion (half_is_normal and
+    normal_to_half in csrc/tge_common.h) gives the recipe's bits for every
+    float that takes it, over all 2^32."""
+    hipcc = "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not available")
+    d = tempfile.mkdtemp(prefix="tge_half_")
+    exe = os.path.join(d, "half_check")
+    try:
+        subprocess.run([hipcc, "-O2", "-std=c++20", "-pthread",
+                        "-I", os.path.join(ROOT, "aegean-tge_amd", "csrc"), "-I", os.path.join(ROOT, "include"),
+                        "-o", exe, os.path.join(HERE, "native", "half_check.cpp")],
+                       check=True, capture_output=True)
+        r = subprocess.run([exe], capture_output=True, text=True)
+        out = json.loads(r.stdout)
+        assert r.returncode == 0 and out["mismatches"] == 0 and out["range_errors"] == 0, (out, r.stderr)
+        assert out["accepted"] == 2 * 0x0F000000, out
+    finally:
+        shutil.rmtree(d, ignore_errors=True)
+
+
 def _rope_inputs(rows, heads, hd, seed):
     rng = np.random.default_rng(seed)
     x = (rng.standard_normal((rows, heads * hd)) * rng.choice([1e-3, 1, 30, 3e4], (rows, 1))
