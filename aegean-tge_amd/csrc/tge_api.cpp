@@ -528,7 +528,7 @@ int tge_batch_plan(tge_batch* b, const tge_kv_pool* pool, const tge_batch_desc* 
   const size_t o_sess = 0;
   const size_t o_tab = align_up(o_sess + st.sessions.size() * sizeof(tge::SessionRec));
   const size_t o_rows = align_up(o_tab + st.tables.size() * sizeof(int));
-  tge::plan::build_append_tiles(st, b->tiles);
+  tge::plan::build_append_tiles(st, b->tiles, pool->desc.format == TGE_KV_I8);
   const size_t o_tiles = align_up(o_rows + st.rows.size() * sizeof(tge::RowRec));
   const size_t o_dec = align_up(o_tiles + b->tiles.size() * sizeof(tge::TileRec));
   AttnPlan& dp = dec ? b->decode : b->prefill;  // (the eager attention plan, if any)

@@ -143,10 +143,12 @@ int build_step(Step& step, int ns, const int* ctx, const int* n_new, const int* 
   return TGE_OK;
 }
 
-void build_append_tiles(const Step& s, std::vector<TileRec>& tiles) {
+void build_append_tiles(const Step& s, std::vector<TileRec>& tiles, bool i8) {
   tiles.clear();
-  const long lanes = (long)s.rows.size() * 2 * s.kv_heads * (s.block_dims / 8);
-  if (s.block_dims <= 64 || lanes * s.block_dims < kAppendPageWork) return;
+  const long values = (long)s.rows.size() * 2 * s.kv_heads * s.block_dims;
+  const int width = s.kv_heads * s.head_dim;  // dims of a row of K
+  if (s.block_dims <= 64 || values / 8 * s.block_dims < kAppendPageWork) return;
+  if (i8 ? width < 256 || values < (width < 1024 ? 9L << 19 : 3L << 20) : width < 1024 && values < 1L << 22) return;
   for (const auto& sr : s.sessions) {
     for (int j = 0; j < sr.n_new;) {
       const int slot = (sr.ctx + j) % kPageTokens;

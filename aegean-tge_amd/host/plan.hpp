@@ -84,15 +84,26 @@ int build_step(Step& step, int n_sessions, const int* ctx, const int* n_new,
 // The step's new rows page by page (TileRec) when its append should store
 // whole pages, empty when it should go row by row. By page a launch has a
 // longer fixed time (four tokens per lane, staged: 5.5-6 us against 4.2) and
-// the better rate, so it takes steps whose lanes (8 values each, in the row
-// kernel) times block width reach 2^26. Row kernel / page kernel, us: 128
-// dims, 4 heads, 2048 rows (2^18 lanes) f16 7.4 / 7.9, int8 6.3 / 6.9; 4096
-// rows 11.6 / 9.2, 9.3 / 8.5; 256 dims, 8 heads, 256 rows (2^17) 6.5 / 7.0,
-// 5.0 / 6.6; 512 rows 9.4 / 7.5, 7.0 / 6.8. 64-dim blocks stay with the row
-// kernel (2 heads, 20,000 rows: int8 9.3 / 10.5), and so do steps whose rows
-// fill their pages to less than three quarters on average.
+// the better rate. The lines are drawn through measured crossings, which lie
+// at fewer values the wider a row is and at more for int8, whose 1-byte
+// stores write half as much. Values here are rows x 2 x KV heads x block
+// width, a row's width its K dims; at least 2^26 / 8 block widths of them
+// (2^22 at 128 dims, 2^21 at 256), and besides: f16 2^22 where a row is
+// narrower than 1024 dims; int8 3 * 2^20, 9 * 2^19 below 1024 dims, none
+// below 256. Row kernel / page kernel, us:
+//   f16   4 x 128, 3584 rows 10.3 / 8.6; 2 x 128, 8192 10.9 / 9.0; 1 x 128,
+//         16384 9.8 / 9.1; 8 x 256, 512 9.4 / 7.2; 4 x 256, 1024 8.1 / 7.2;
+//         past the line 2 x 256, 2048 7.4 / 7.5; 4 x 224, 1024 8.1 / 8.5;
+//         1 x 256, 4096 6.9 / 7.5; 4 x 128, 2048 7.3 / 7.6
+//   int8  8 x 256, 768 8.7 / 8.0; 8 x 128, 2048 9.9 / 8.5; 4 x 128, 5000
+//         (a part of a page last) 10.2 / 10.3, 8192 17.6 / 15.4; 2 x 128,
+//         12000 10.8 / 10.7; past the line 8 x 256, 512 6.7 / 6.8; 2 x 256,
+//         2048 5.7 / 6.8; 1 x 128, 16384 7.7 / 8.5, 32768 14.4 / 15.4
+// 64-dim blocks stay with the row kernel (2 heads, 20,000 rows: int8 9.3 /
+// 10.5, f16 11.5 / 10.8 with a page kernel for them), and so do steps whose
+// rows fill their pages to less than three quarters on average.
 constexpr long kAppendPageWork = 1L << 26;
-void build_append_tiles(const Step& s, std::vector<TileRec>& tiles);
+void build_append_tiles(const Step& s, std::vector<TileRec>& tiles, bool i8 = false);
 
 // Work lists of one attention kind for the current step.
 struct AttnLists {

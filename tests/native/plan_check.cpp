@@ -616,7 +616,7 @@ int describe(int argc, char** argv) {
     prefill_ns = std::min<long>(prefill_ns, std::chrono::nanoseconds(t2 - t1).count());
   }
   std::vector<TileRec> tiles;
-  build_append_tiles(st, tiles);
+  build_append_tiles(st, tiles, a[3] != 0);
   std::printf("items %zu parts %d tile_rows %d append_pages %zu step_ns %ld prefill_ns %ld\n", pf.work.size(), pf.parts,
               pf.tile_rows, tiles.size(), step_ns, prefill_ns);
   return 0;

@@ -9,7 +9,7 @@ import pytest
 import oracle as O
 import synth
 import tge_kv as tk
-from _paged import PAGE_APPEND_STEP, PAGE_APPENDS, PREFILL_PLANS, PagedCase
+from _paged import PAGE_APPEND_STEP, PAGE_APPENDS, PREFILL_PLANS, ROW_APPENDS, PagedCase
 from _util import assert_attention_close, bits
 
 pytestmark = pytest.mark.gpu
@@ -1004,11 +1004,12 @@ def test_random_append_bitexact(gpu, i):
     case.close()
 
 
-@pytest.mark.parametrize("fmt,sf,kvh,hd", PAGE_APPENDS)
+@pytest.mark.parametrize("fmt,sf,kvh,hd", PAGE_APPENDS + ROW_APPENDS)
 def test_append_whole_pages_bitexact(gpu, fmt, sf, kvh, hd):
-    """A step of many rows stores page by page: sessions that start at, after
-    and before a page edge, whole pages, pages shared with earlier rows and
-    a last wave that is not full; special values among them."""
+    """A step of many rows stores page by page (test_host_plan.py: which
+    do): sessions that start at, after and before a page edge, whole pages,
+    pages shared with earlier rows and a last wave that is not full; special
+    values among them."""
     case = PagedCase(kvh * 2, kvh, hd, fmt, *PAGE_APPEND_STEP, scale_format=sf, seed=31,
                      outlier_frac=0.01 if fmt == tk.KV_I8 else 0)
     rng = np.random.default_rng(5)
