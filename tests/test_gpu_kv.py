@@ -398,7 +398,7 @@ def test_prefill_chunks_match_oracle(gpu):
 # Block prefill at head_dim 128 in both tile widths: (q_heads, kv_heads,
 # format, contexts, n_new). On 256 compute units the planner takes 280
 # unsplit 64-row tiles for the first two, 136 unsplit 64-row tiles (f16) or
-# 68 128-row tiles in two pieces each (int8) for the next, and 56 64-row
+# 68 128-row tiles in two pieces each (int8) for the next, and 108 64-row
 # tiles for the small step. (PREFILL_PLANS has launches of whole 128-row
 # tiles.)
 TILE_CASES = {
