@@ -19,8 +19,8 @@ struct LaneCodes {
   float scale;
 };
 
-// Encode one lane's 8 values. f16: each value with the reference's
-// float_to_half recipe. int8: the four lanes of the block (adjacent,
+// Encode one lane's 8 values. f16: each value with the bits of
+// the reference's float_to_half recipe. int8: the four lanes of the block (adjacent,
 // aligned to 4 in the wave) combine their absmax runs in order (see
 // FoldRun), then each computes the block's scale and inverse exactly as
 // quantize_kv_block does (correctly rounded fp32 division) and quantizes
@@ -30,19 +30,8 @@ template <int FMT>
 __device__ __forceinline__ LaneCodes encode_lane(const float (&x)[8]) {
   LaneCodes c{{0, 0, 0, 0}, 0.0f};
   if (FMT == kF16) {
-    // Normal halves need no branch; a lane with any other value takes the
-    // recipe for all eight.
-    bool normal = true;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) normal = normal && half_is_normal(x[i]);
-    if (normal) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) c.w[i >> 1] |= (uint32_t)normal_to_half(x[i]) << (16 * (i & 1));
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        c.w[i] = float_to_half_ref(x[2 * i]) | ((uint32_t)float_to_half_ref(x[2 * i + 1]) << 16);
-    }
+    for (int i = 0; i < 4; ++i) c.w[i] = any_to_half(x[2 * i]) | any_to_half(x[2 * i + 1]) << 16;
   } else {
     // the block's absmax: lane runs joined in lane order
     const FoldRun mine = fold_run(x);

@@ -121,16 +121,27 @@ __host__ __device__ inline uint16_t float_to_half_ref(float value) {
   return (uint16_t)(sign | (kept + ((frac >> 12) & 1u)));
 }
 
-// The recipe without a branch for magnitudes from 2^-14 up to 65536: with t
-// the magnitude's bits, the kept mantissa plus the guard bit is
-// (t + 2^12) >> 13, less the exponents' offset (a carry out of the largest
-// half gives infinity, as the recipe does).
-__host__ __device__ inline bool half_is_normal(float value) {
-  return (f32_as_u32(value) & 0x7FFFFFFFu) - 0x38800000u < 0x0F000000u;
+// f16 bits of the float with bits u, rounded to nearest even.
+__host__ __device__ inline uint32_t half_bits_rne(uint32_t u) {
+  float x;
+  __builtin_memcpy(&x, &u, 4);
+  const _Float16 h = (_Float16)x;
+  uint16_t bits;
+  __builtin_memcpy(&bits, &h, 2);
+  return bits;
 }
-__host__ __device__ inline uint32_t normal_to_half(float value) {
-  const uint32_t u = f32_as_u32(value);
-  return ((((u & 0x7FFFFFFFu) + 0x1000u) >> 13) - 0x1C000u) | ((u >> 16) & 0x8000u);
+
+// The recipe's bits for any float, without branches: the appends' f16 encoder
+// (with branches, values of different kinds in a wave take one path after the
+// other). The conversion to nearest even gives the recipe's bits once the
+// lowest mantissa bit is set, which puts exact ties above the middle and moves
+// no other value across one; below 2^-24 the recipe flushes, and infinities
+// and NaNs are selected.
+__host__ __device__ inline uint32_t any_to_half(float value) {
+  const uint32_t u = f32_as_u32(value), t = (u & 0x7FFFFFFFu) | 1u;
+  uint32_t h = t < 0x33800000u ? 0u : half_bits_rne(t);
+  h = t >= 0x7F800000u ? (value != value ? 0x7E00u : 0x7C00u) : h;
+  return h | ((u >> 16) & 0x8000u);
 }
 
 // static_cast<int>(float) as the reference's x86-64 build executes it

@@ -453,10 +453,9 @@ def test_split_absmax_fold_matches_sequential():
         shutil.rmtree(d, ignore_errors=True)
 
 
-def test_normal_half_path_matches_recipe():
-    """The append's branch-free f16 conversion (half_is_normal and
-    normal_to_half in csrc/tge_common.h) gives the recipe's bits for every
-    float that takes it, over all 2^32."""
+def test_append_half_conversion_matches_recipe():
+    """The appends' f16 conversion (any_to_half, csrc/tge_common.h) gives the
+    recipe's bits over all 2^32 floats."""
     hipcc = "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         pytest.skip("hipcc not available")
@@ -469,8 +468,7 @@ def test_normal_half_path_matches_recipe():
                        check=True, capture_output=True)
         r = subprocess.run([exe], capture_output=True, text=True)
         out = json.loads(r.stdout)
-        assert r.returncode == 0 and out["mismatches"] == 0 and out["range_errors"] == 0, (out, r.stderr)
-        assert out["accepted"] == 2 * 0x0F000000, out
+        assert r.returncode == 0 and out["mismatches"] == 0, (out, r.stderr)
     finally:
         shutil.rmtree(d, ignore_errors=True)
 
