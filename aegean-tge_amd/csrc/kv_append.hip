@@ -55,10 +55,10 @@ __global__ __launch_bounds__(256) void kv_append_kernel(AppendParams p) {
 // contiguous KiB per store. Pages that the step writes in part store element
 // by element, as the row kernel does.
 // The row kernel is bound by its 1- and 2-byte V stores. 20,000 rows, row
-// kernel -> this one: 4 heads of 128 dims int8 38.8 -> 28.5 us (104 MB: 3.7
-// TB/s, of which 5.5-6 us are a launch's fixed time), f16 44.7 -> 27.9 us (123
-// MB: 4.4 TB/s); 8 heads of 256 dims int8 174 -> 88 us, f16 226 -> 91 us (492
-// MB: 5.4 TB/s).
+// kernel -> this one: 4 heads of 128 dims int8 39.4 -> 27.9 us (104 MB: 3.7
+// TB/s, of which 6 us are a launch's fixed time), f16 45.6 -> 27.5 us (123 MB:
+// 4.5 TB/s); 8 heads of 256 dims int8 182 -> 86 us, f16 230 -> 90 us (492 MB:
+// 5.5 TB/s).
 template <int FMT>
 __global__ __launch_bounds__(256) void kv_append_pages_kernel(AppendParams p) {
   constexpr int E = FMT == kF16 ? 2 : 1;

@@ -147,8 +147,9 @@ void build_append_tiles(const Step& s, std::vector<TileRec>& tiles, bool i8) {
   tiles.clear();
   const long values = (long)s.rows.size() * 2 * s.kv_heads * s.block_dims;
   const int width = s.kv_heads * s.head_dim;  // dims of a row of K
-  if (s.block_dims <= 64 || values / 8 * s.block_dims < kAppendPageWork) return;
-  if (i8 ? width < 256 || values < (width < 1024 ? 9L << 19 : 3L << 20) : width < 1024 && values < 1L << 22) return;
+  const bool wide = width >= 1024;
+  const long line = i8 ? (wide ? 3L << 20 : 9L << 19) : (wide ? 1L << 20 : 2L << 20);
+  if (s.block_dims <= 64 || values < line || (i8 && width < 256)) return;
   for (const auto& sr : s.sessions) {
     for (int j = 0; j < sr.n_new;) {
       const int slot = (sr.ctx + j) % kPageTokens;

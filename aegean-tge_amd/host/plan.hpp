@@ -83,26 +83,27 @@ int build_step(Step& step, int n_sessions, const int* ctx, const int* n_new,
 
 // The step's new rows page by page (TileRec) when its append should store
 // whole pages, empty when it should go row by row. By page a launch has a
-// longer fixed time (four tokens per lane, staged: 5.5-6 us against 4.2) and
-// the better rate. The lines are drawn through measured crossings, which lie
-// at fewer values the wider a row is and at more for int8, whose 1-byte
-// stores write half as much. Values here are rows x 2 x KV heads x block
-// width, a row's width its K dims; at least 2^26 / 8 block widths of them
-// (2^22 at 128 dims, 2^21 at 256), and besides: f16 2^22 where a row is
-// narrower than 1024 dims; int8 3 * 2^20, 9 * 2^19 below 1024 dims, none
-// below 256. Row kernel / page kernel, us:
-//   f16   4 x 128, 3584 rows 10.3 / 8.6; 2 x 128, 8192 10.9 / 9.0; 1 x 128,
-//         16384 9.8 / 9.1; 8 x 256, 512 9.4 / 7.2; 4 x 256, 1024 8.1 / 7.2;
-//         past the line 2 x 256, 2048 7.4 / 7.5; 4 x 224, 1024 8.1 / 8.5;
-//         1 x 256, 4096 6.9 / 7.5; 4 x 128, 2048 7.3 / 7.6
-//   int8  8 x 256, 768 8.7 / 8.0; 8 x 128, 2048 9.9 / 8.5; 4 x 128, 5000
-//         (a part of a page last) 10.2 / 10.3, 8192 17.6 / 15.4; 2 x 128,
-//         12000 10.8 / 10.7; past the line 8 x 256, 512 6.7 / 6.8; 2 x 256,
-//         2048 5.7 / 6.8; 1 x 128, 16384 7.7 / 8.5, 32768 14.4 / 15.4
+// longer fixed time (four tokens per lane, staged: f16 4.9 us, int8 6.0,
+// against 3.8-4.2) and the better rate. The lines are drawn through measured
+// crossings, which lie at fewer values the wider a row is and at more for
+// int8, whose 1-byte stores write half as much. Values here are rows x 2 x KV
+// heads x block width, a row's width its K dims: f16 from 2^20 values on, 2^21
+// where a row is narrower than 1024 dims; int8 from 3 * 2^20, 9 * 2^19 below
+// 1024 dims, never below 256. Row kernel / page kernel, us:
+//   f16   8 x 256, 257 rows 6.3 / 4.8; 8 x 128, 513 5.4 / 4.8; 4 x 128, 2048
+//         7.4 / 5.7; 2 x 128, 4097 6.6 / 5.5; 1 x 128, 8200 6.1 / 5.7; 1 x
+//         256, 4100 6.7 / 5.8; below the line 4 x 128, 1100 (a part of a
+//         page last) 5.1 / 5.6, 1500 5.8 / 5.9; 1 x 128, 6000 4.9 / 5.3
+//   int8  8 x 256, 768 8.9 / 8.0; 8 x 128, 2048 9.9 / 8.5; 4 x 128, 5000
+//         10.2 / 10.3, 8192 17.6 / 15.3; 2 x 128, 12000 10.8 / 10.8; below
+//         the line 8 x 256, 512 6.7 / 6.7; 2 x 256, 2048 5.7 / 6.9; 1 x 128,
+//         16384 7.8 / 8.5, 32768 14.3 / 15.4
 // 64-dim blocks stay with the row kernel (2 heads, 20,000 rows: int8 9.3 /
-// 10.5, f16 11.5 / 10.8 with a page kernel for them), and so do steps whose
-// rows fill their pages to less than three quarters on average.
-constexpr long kAppendPageWork = 1L << 26;
+// 10.5, f16 11.5 / 10.8 with a page kernel for them and an earlier f16
+// encoder), and so do steps whose rows fill their pages to less than three
+// quarters on average. No line lies below kAppendPageWork lanes (8 values
+// each) times block width.
+constexpr long kAppendPageWork = 1L << 24;
 void build_append_tiles(const Step& s, std::vector<TileRec>& tiles, bool i8 = false);
 
 // Work lists of one attention kind for the current step.

@@ -25,12 +25,12 @@ PREFILL_PLANS = {
     "cut_96_narrow_i8": (16, 4, 96, tk.KV_I8, 1536, 512, "cut", 64),
 }
 # A step and the (format, scale format, KV heads, head_dim) at which its
-# append goes page by page, and narrower ones at which it goes row by row.
+# append goes page by page, and a narrower one at which it goes row by row.
 PAGE_APPEND_STEP = ([0, 16, 21, 500, 15], [1600, 1024, 1115, 533, 769])
 PAGE_APPENDS = [
-    (tk.KV_F16, 0, 5, 100), (tk.KV_F16, 0, 4, 128), (tk.KV_F16, 0, 2, 256), (tk.KV_F16, 0, 2, 132),
+    (tk.KV_F16, 0, 5, 100), (tk.KV_F16, 0, 4, 128), (tk.KV_F16, 0, 1, 256), (tk.KV_F16, 0, 2, 132),
     (tk.KV_I8, 1, 5, 96), (tk.KV_I8, 0, 4, 128), (tk.KV_I8, 1, 2, 256), (tk.KV_I8, 0, 4, 224)]
-ROW_APPENDS = [(tk.KV_F16, 0, 1, 256), (tk.KV_I8, 0, 1, 224)]
+ROW_APPENDS = [(tk.KV_I8, 0, 1, 224)]
 
 
 class PagedCase:

@@ -72,9 +72,10 @@ def test_append_by_page_where_it_gains(tmp_path):
     store row by row (KV heads, head_dim, int8, rows), those at which the
     page kernel did store by page."""
     by_row = [(2, 256, 1, 2048), (1, 128, 1, 16384), (1, 128, 1, 32768), (4, 256, 1, 1024), (8, 256, 1, 512),
-              (2, 256, 0, 2048), (4, 224, 0, 1024), (1, 256, 0, 4096), (4, 128, 0, 2048), (4, 128, 1, 3072)]
+              (4, 128, 1, 3072), (4, 128, 0, 1100), (4, 128, 0, 1500), (2, 128, 0, 2600), (1, 128, 0, 6000)]
     by_page = [(8, 256, 1, 1024), (8, 128, 1, 2048), (4, 128, 1, 8192), (4, 256, 1, 2048), (2, 256, 1, 6144),
-               (8, 256, 0, 512), (4, 256, 0, 1024), (4, 128, 0, 4096), (2, 128, 0, 8192), (1, 128, 0, 16384)]
+               (8, 256, 0, 257), (8, 128, 0, 513), (4, 256, 0, 515), (4, 128, 0, 2048), (2, 128, 0, 4097),
+               (1, 128, 0, 8200), (2, 256, 0, 2048), (1, 256, 0, 4100)]
     out = build_and_run(tmp_path, "plan_check", ["aegean-tge_amd/host/plan.cpp", "tests/native/plan_check.cpp"],
                         [(kvh, kvh, hd, i8, 0, n) for kvh, hd, i8, n in by_row + by_page])
     for case, line in zip(by_row + by_page, out.splitlines()):
