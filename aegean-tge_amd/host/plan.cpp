@@ -359,7 +359,7 @@ void add_units(std::vector<WorkRec>& work, std::vector<int>& at, std::vector<Red
 // by kernel: the launch, an item's start and end, and a page of an item.
 // Where a compute unit holds three workgroups (64 dims), `page` is that of
 // an item alone there, and `two` and `three` times as much is a page of each
-// of two or three that share it. Fitted to 1,318 launches (12 to 1,500
+// of two or three that share it. Fitted to 1,636 launches (12 to 2,826
 // items, 28/4, 12/2, 16/4 x 96, 14/2 x 64 and 16/8 x 256 heads, contexts up
 // to 24,000): 5 to 6 % rms off at 128 and 256 dims, 8 to 9 % at 64.
 struct PrefillCost {
@@ -374,7 +374,7 @@ PrefillCost prefill_cost(int block_dims, int tile_rows, bool i8) {
   if (tile_rows == 64) return i8 ? PrefillCost{3.6, 6.1, 0.333, 1, 1, 1} : PrefillCost{3.3, 6.1, 0.167, 1, 1, 1};
   return i8 ? PrefillCost{3.5, 9.9, 0.422, 1, 1, 1} : PrefillCost{3.2, 10.0, 0.230, 1, 1, 1};
 }
-// The merge launch behind it, and 64 KiB of partials through it (1,300
+// The merge launch behind it, and 64 KiB of partials through it (1,368
 // launches, 0.9 us rms off).
 constexpr double kMergeLaunch = 5.6, kMergePart = 0.0100;
 
